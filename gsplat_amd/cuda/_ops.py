@@ -1025,7 +1025,8 @@ class RasterReplay:
 # Largest replay workspace (bytes) one rasterizer call may allocate.  The
 # records take 16 (1 + C) bytes per intersection for C channels (a record of
 # T and the C colour sums for each of a tile's pixels at every 64th
-# intersection of its range), allocated for the whole range although only the
+# intersection of its range; T alone, 16 bytes, for more than eight channels
+# from 3,072 16x16 tiles on), allocated for the whole range although only the
 # boundaries a pixel is still active at are written.  Above this budget the
 # forward keeps no replay state and the backward replays whole tiles from the
 # final transmittance (gsplat_rasterize_bwd), as the reference does.
