@@ -22,10 +22,11 @@ _P = c_void_p
 # of include/gsplat_hip.h.  load() refuses a library built from any other
 # header, and a CPU test keeps this digest and _SIGNATURES equal to the
 # header's.  Change all three together.
-_ABI_VERSION = "0ed8ce82e6221bc5"
+_ABI_VERSION = "1699fda273b66910"
 
 # name -> argtypes (restype int unless listed in _RESTYPES)
 _SIGNATURES = {
+    "gsplat_wait_count": [_P, _P, _P],
     "gsplat_last_error": [],
     "gsplat_version": [],
     "gsplat_abi_version": [],
@@ -287,6 +288,21 @@ def call(name: str, *args) -> None:
     if rc != 0:
         msg = lib.gsplat_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed ({rc}): {msg}")
+
+
+def host_count() -> torch.Tensor:
+    """A pinned host word for a kernel to write a count into, holding -1."""
+    word = torch.empty(1, dtype=torch.int64, pin_memory=True)
+    c_int64.from_address(word.data_ptr()).value = -1
+    return word
+
+
+def wait_count(word: torch.Tensor, stream_handle: int) -> int:
+    """The count a kernel queued on the stream writes into ``word``
+    (host_count), as soon as it is there."""
+    value = c_int64()
+    call("gsplat_wait_count", word.data_ptr(), ctypes.addressof(value), stream_handle)
+    return value.value
 
 
 def query(name: str, *args) -> int:

@@ -51,6 +51,37 @@ extern "C" const char *gsplat_version(void) {
     return "gsplat_hip 0.1.0 gfx950";
 }
 
+extern "C" int gsplat_wait_count(const int64_t *word, int64_t *value,
+                                 gsplat_stream_t stream) {
+    gs::clear_error();
+    GS_REQUIRE(word != nullptr && value != nullptr, "wait_count: NULL word or value");
+    for (uint32_t spin = 1;; ++spin) {
+        const int64_t v = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (v >= 0) {
+            *value = v;
+            return GSPLAT_OK;
+        }
+        if ((spin & 4095u) != 0) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        const hipError_t err = hipStreamQuery(gs::as_stream(stream));
+        if (err == hipErrorNotReady)
+            continue;
+        (void)hipGetLastError();
+        if (err != hipSuccess)
+            return gs::fail(GSPLAT_ERR_LAUNCH,
+                            std::string("wait_count: ") + hipGetErrorString(err));
+        // the stream has drained: the word is written now, or never
+        const int64_t last = __atomic_load_n(word, __ATOMIC_ACQUIRE);
+        if (last < 0)
+            return gs::fail(GSPLAT_ERR_INVALID_ARGUMENT,
+                            "wait_count: nothing queued on the stream writes the word");
+        *value = last;
+        return GSPLAT_OK;
+    }
+}
+
 // The build passes the digest of include/gsplat_hip.h's declarations.
 #ifndef GSPLAT_ABI_HASH
 #error "GSPLAT_ABI_HASH must be defined by the build (digest of include/gsplat_hip.h)"

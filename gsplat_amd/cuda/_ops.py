@@ -21,7 +21,7 @@ from typing import Optional, Tuple
 import torch
 from torch import Tensor
 
-from .._lib import AdamTensor, call, check_input, ptr, query
+from .._lib import AdamTensor, call, check_input, host_count, ptr, query, wait_count
 
 _F32 = torch.float32
 _I32 = torch.int32
@@ -29,7 +29,9 @@ _I64 = torch.int64
 
 
 def _stream(t: Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the current stream of t's device (torch.cuda.current_stream
+    without its Stream object: 7 us a call, six calls a step)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _prod(shape) -> int:
@@ -360,7 +362,7 @@ def packed_front_fwd(
         # the kernel writes the visible count straight into pinned host
         # memory (device-accessible at the same address), so no copy kernel
         # sits on the stream between the projection and the colours
-        nnz_host = torch.empty(1, dtype=_I64, pin_memory=True)
+        nnz_host = host_count()
         call("gsplat_projection_packed_fwd", B, C, N, ptr(means), ptr(covars),
              ptr(quats), ptr(scales), ptr(opacities), ptr(viewmats), ptr(Ks),
              int(image_width), int(image_height), float(eps2d),
@@ -369,8 +371,6 @@ def packed_front_fwd(
              ptr(batch_ids), ptr(camera_ids), ptr(gaussian_ids), ptr(radii),
              ptr(means2d), ptr(depths), ptr(conics), ptr(comps), ptr(nnz_host),
              ptr(row_of), ptr(row_opac), st)
-        copied = torch.cuda.Event()
-        copied.record()
         I = B * C
         tile_first = isect is not None and (
             int(I).bit_length()
@@ -401,8 +401,7 @@ def packed_front_fwd(
         else:
             call("gsplat_sh_rows_fwd", B, C, N, K, int(sh_degree), ptr(means),
                  ptr(viewmats), ptr(features), ptr(row_of), ptr(row_colors), st)
-        copied.synchronize()
-        nnz = int(nnz_host[0])
+        nnz = wait_count(nnz_host, st)
         if isect is not None and nnz > 0:
             ts, tw, th = isect["tile_size"], isect["tile_width"], isect["tile_height"]
             if tile_first:
@@ -803,6 +802,15 @@ def intersect_tile(
         state = isect_prepare_sorted(means2d, radii, depths, conics, opacities, img,
                                      N, I, tile_size, tile_width, tile_height,
                                      tiles_per_gauss)
+        # as in the packed front end, the second stage is queued before the
+        # host knows the count, sized from the last call of the same shape,
+        # so that the GPU does not wait for the host in between
+        shape = (dev.index, n, packed, int(I), int(tile_size), int(tile_width),
+                 int(tile_height))
+        state["shape"] = shape
+        last = _ISECT_SHAPES.get(shape)
+        if last is not None:
+            isect_emit_sorted_queue(state, last + last // 16 + 4096)
         return isect_emit_sorted(state)[:3]
     cum = torch.empty(n, dtype=_I64, device=dev)
     ws = torch.empty(query("gsplat_isect_count_workspace_size", n),
@@ -826,6 +834,8 @@ def intersect_tile(
 # call queues its emission for this many plus 1/16 (and 4096) before the
 # host knows its own count.
 _ISECT_LAST = {}
+# The same for intersect_tile, per shape of the call (at most 64 of them).
+_ISECT_SHAPES = {}
 
 
 def isect_capacity(device: torch.device) -> Optional[int]:
@@ -860,8 +870,8 @@ def isect_prepare_sorted(means2d, radii, depths, conics, opacities, img, N, I,
     """First half of the sorted intersection of n > 0 rows (inputs checked by
     the caller): the tile counts, the rows' first slots in row order and
     their sweep records (gsplat_isect_prepare_rows).  The intersection count
-    goes to a pinned host word behind an event, so the caller can queue or
-    do other work before ``isect_emit_sorted`` waits for it."""
+    goes to a pinned host word, so the caller can queue or do other work
+    before ``isect_emit_sorted`` waits for it."""
     n = means2d.numel() // 2
     dev = means2d.device
     st = _stream(means2d)
@@ -874,7 +884,7 @@ def isect_prepare_sorted(means2d, radii, depths, conics, opacities, img, N, I,
         "records": torch.empty(n, 8, dtype=_F32, device=dev),
     }
     # the count goes straight into pinned host memory (no copy kernel)
-    host = torch.empty(1, dtype=_I64, pin_memory=True)
+    host = host_count()
     ws = torch.empty(query("gsplat_isect_prepare_rows_workspace_size", n),
                      dtype=torch.uint8, device=dev)
     call("gsplat_isect_prepare_rows", n, N, ptr(img), ptr(means2d), ptr(radii),
@@ -882,9 +892,7 @@ def isect_prepare_sorted(means2d, radii, depths, conics, opacities, img, N, I,
          int(tile_width), int(tile_height), ptr(ws), ws.numel(),
          ptr(tiles_per_gauss), ptr(state["row_starts"]), ptr(state["records"]),
          ptr(host), st)
-    ev = torch.cuda.Event()
-    ev.record()
-    state["total"] = (host, ev)
+    state["total"] = (host, st)
     return state
 
 
@@ -903,12 +911,11 @@ def isect_prepare_counted(counted, means2d, radii, depths, conics, opacities, im
         "row_starts": counted["row_starts"][:n + 1],
         "records": counted["records"][:n],
     }
-    host = torch.empty(1, dtype=_I64, pin_memory=True)
+    host = host_count()
+    st = _stream(means2d)
     call("gsplat_isect_row_starts", n, ptr(counted["ws"]), counted["ws"].numel(),
-         ptr(state["row_starts"]), ptr(host), _stream(means2d))
-    ev = torch.cuda.Event()
-    ev.record()
-    state["total"] = (host, ev)
+         ptr(state["row_starts"]), ptr(host), st)
+    state["total"] = (host, st)
     return state
 
 
@@ -917,11 +924,14 @@ def isect_emit_sorted(state):
     intersections in row order, sorts them on the image|tile bits and every
     tile's rows on their depth bits (gsplat_isect_emit_tiles).  Returns
     (tiles_per_gauss, isect_ids, flatten_ids, isect_offsets [I, th, tw])."""
-    host, ev = state["total"]
-    ev.synchronize()
-    n_isects = int(host[0])
+    n_isects = wait_count(*state["total"])
     dev = state["means2d"].device
-    _ISECT_LAST[dev.index] = n_isects
+    if "shape" in state:
+        if len(_ISECT_SHAPES) >= 64:
+            _ISECT_SHAPES.clear()
+        _ISECT_SHAPES[state["shape"]] = n_isects
+    else:
+        _ISECT_LAST[dev.index] = n_isects
     queued = state.get("queued")
     if queued is not None and n_isects <= queued[0]:
         return (state["tiles_per_gauss"], queued[1][:n_isects], queued[2][:n_isects],

@@ -49,6 +49,15 @@ enum {
     GSPLAT_CAMERA_FISHEYE = 2,
 };
 
+/* Waits until the host word `word` (pinned, device-visible memory that a
+ * kernel queued on `stream` writes a count >= 0 into: nnz_out, n_isects_out)
+ * no longer holds the negative value the caller put there before the launch,
+ * and returns it in *value.  Polls the word, so the host goes on as soon as
+ * the count arrives instead of when an event behind the kernel has been
+ * processed; the stream is queried now and then, and a stream that failed or
+ * drained without the word having been written is an error. */
+int gsplat_wait_count(const int64_t *word, int64_t *value, gsplat_stream_t stream);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char *gsplat_last_error(void);
 
