@@ -363,9 +363,22 @@ __global__ void __launch_bounds__(kProjThreads)
 // them short (245 links per million rows).
 constexpr int kPackThreads = 1024;
 constexpr int kPackItems = 4;
-constexpr int kPackRows = kPackThreads * kPackItems;
 
-template <bool COVARS>
+// Rows of a workgroup.  4,096-row workgroups reach fewer than 256 CUs below a
+// million rows, and a few of them only at small scenes, where the time is one
+// workgroup's own latency: up to kPackSmall rows workgroups of 256 threads
+// take one row each.  10,000 rows 18.2 -> 6.9 us, 60,000 20.6 -> 9.7, 150,000
+// 21.6 -> 18.1, 300,000 23.2 -> 33.9 (their look-back chain is 16 times as
+// long): the line is at half a look-back window of small workgroups per CU.
+constexpr int64_t kPackSmall = 131072;
+
+constexpr int kPackSmallThreads = 256;
+constexpr int64_t kPackLargeRows = kPackThreads * kPackItems;
+constexpr int64_t pack_rows(int64_t rows) {
+    return rows <= kPackSmall ? kPackSmallThreads : kPackLargeRows;
+}
+
+template <bool COVARS, int kPackThreads, int kPackItems>
 __global__ void __launch_bounds__(kPackThreads) projection_packed_fwd_kernel(
     const FwdArgs a, Lookback lb, int32_t *__restrict__ indptr,
     int64_t *__restrict__ batch_ids, int64_t *__restrict__ camera_ids,
@@ -375,6 +388,7 @@ __global__ void __launch_bounds__(kPackThreads) projection_packed_fwd_kernel(
     int64_t *__restrict__ nnz_out, int32_t *__restrict__ row_of,
     float *__restrict__ row_opacities) {
     constexpr int NW = kPackThreads / kWave;
+    constexpr int kPackRows = kPackThreads * kPackItems;
     static_assert(kPackItems * NW <= kWave, "one wave scans the wave counts");
     __shared__ uint32_t s_ticket;
     __shared__ uint32_t s_cnt[kPackItems * NW];  // survivors per (slice, wave)
@@ -1395,14 +1409,14 @@ extern "C" int gsplat_projection_fused_fwd(
 
 extern "C" size_t gsplat_projection_packed_workspace_size(int64_t B, int64_t C,
                                                           int64_t N) {
-    return lookback_bytes(ceil_div(B * C * N, kPackRows));
+    return lookback_bytes(ceil_div(B * C * N, pack_rows(B * C * N)));
 }
 
 namespace gs {
 namespace {
 
 // The packed forward over a caller-checked look-back workspace of at least
-// lookback_bytes(ceil(B*C*N / kPackRows)) bytes.
+// lookback_bytes(ceil(B*C*N / pack_rows(B*C*N))) bytes.
 int packed_fwd_launch(int64_t B, int64_t C, int64_t N, const float *means,
                       const float *covars, const float *quats, const float *scales,
                       const float *opacities, const float *viewmats, const float *Ks,
@@ -1414,22 +1428,30 @@ int packed_fwd_launch(int64_t B, int64_t C, int64_t N, const float *means,
                       float *compensations, int64_t *nnz_out, int32_t *row_of,
                       float *row_opacities, hipStream_t st) {
     const int64_t rows = B * C * N;
-    const int64_t blocks = ceil_div(rows, kPackRows);
+    const int64_t blocks = ceil_div(rows, pack_rows(rows));
     GS_TRY(clear_lookback(workspace, blocks, st));
     FwdArgs a{B, C, N, means, covars, quats, scales, opacities, viewmats, Ks,
               (float)image_width, (float)image_height, eps2d, near_plane,
               far_plane, radius_clip, camera_model, compensations != nullptr,
               rows < (int64_t(1) << 31)};
-    if (covars != nullptr)
-        projection_packed_fwd_kernel<true><<<(unsigned)blocks, kPackThreads, 0, st>>>(
-            a, lookback_from(workspace), indptr, batch_ids, camera_ids,
-            gaussian_ids, radii, means2d, depths, conics, compensations,
-            nnz_out, row_of, row_opacities);
-    else
-        projection_packed_fwd_kernel<false><<<(unsigned)blocks, kPackThreads, 0, st>>>(
-            a, lookback_from(workspace), indptr, batch_ids, camera_ids,
-            gaussian_ids, radii, means2d, depths, conics, compensations,
-            nnz_out, row_of, row_opacities);
+#define GS_PACK(COVARS, THREADS, ITEMS)                                        \
+    projection_packed_fwd_kernel<COVARS, THREADS, ITEMS>                       \
+        <<<(unsigned)blocks, THREADS, 0, st>>>(                                \
+            a, lookback_from(workspace), indptr, batch_ids, camera_ids,        \
+            gaussian_ids, radii, means2d, depths, conics, compensations,       \
+            nnz_out, row_of, row_opacities)
+    if (rows <= kPackSmall) {
+        if (covars != nullptr)
+            GS_PACK(true, kPackSmallThreads, 1);
+        else
+            GS_PACK(false, kPackSmallThreads, 1);
+    } else {
+        if (covars != nullptr)
+            GS_PACK(true, kPackThreads, kPackItems);
+        else
+            GS_PACK(false, kPackThreads, kPackItems);
+    }
+#undef GS_PACK
     return check_launch("projection_packed_fwd_kernel");
 }
 
@@ -1458,7 +1480,7 @@ int check_packed_fwd(int64_t B, int64_t C, int64_t N, const float *means,
 }
 
 // Scratch of the allocation-free packed forward: the look-back ticket and
-// status words of up to kNoAllocMaxBlocks workgroups (kPackRows rows each).
+// status words of up to kNoAllocMaxBlocks workgroups (kPackLargeRows rows each).
 // Each device holds its own copy for the life of the process; host code
 // reaches it only through the address hipGetSymbolAddress returns on that
 // device (the symbol's name is a host-side stand-in).
@@ -1516,7 +1538,7 @@ extern "C" int gsplat_projection_packed_fwd(
                             Ks, image_width, image_height, camera_model, indptr,
                             batch_ids, camera_ids, gaussian_ids, radii, means2d, depths,
                             conics, nnz_out, row_opacities));
-    const int64_t blocks = ceil_div(B * C * N, kPackRows);
+    const int64_t blocks = ceil_div(B * C * N, pack_rows(B * C * N));
     GS_REQUIRE(workspace != nullptr && workspace_bytes >= lookback_bytes(blocks),
                "projection_packed: workspace too small");
     return packed_fwd_launch(B, C, N, means, covars, quats, scales, opacities, viewmats,
@@ -1528,7 +1550,7 @@ extern "C" int gsplat_projection_packed_fwd(
 }
 
 extern "C" int64_t gsplat_projection_packed_fwd_noalloc_max_rows(void) {
-    return kNoAllocMaxBlocks * kPackRows;
+    return kNoAllocMaxBlocks * kPackLargeRows;
 }
 
 extern "C" int gsplat_projection_packed_fwd_noalloc(
@@ -1545,12 +1567,12 @@ extern "C" int gsplat_projection_packed_fwd_noalloc(
                             Ks, image_width, image_height, camera_model, indptr,
                             batch_ids, camera_ids, gaussian_ids, radii, means2d, depths,
                             conics, nnz_out, row_opacities));
-    const int64_t blocks = ceil_div(B * C * N, kPackRows);
+    const int64_t blocks = ceil_div(B * C * N, pack_rows(B * C * N));
     if (blocks > kNoAllocMaxBlocks)
         return fail(GSPLAT_ERR_WORKSPACE,
                     "projection_packed_fwd_noalloc: " + std::to_string(B * C * N) +
                         " rows exceed the static scratch's limit of " +
-                        std::to_string(kNoAllocMaxBlocks * kPackRows) + " rows");
+                        std::to_string(kNoAllocMaxBlocks * kPackLargeRows) + " rows");
     void *ws = nullptr;
     GS_TRY(device_scratch(&ws));
     return packed_fwd_launch(B, C, N, means, covars, quats, scales, opacities, viewmats,
