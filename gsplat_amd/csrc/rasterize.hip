@@ -936,11 +936,15 @@ __device__ __forceinline__ void rasterize_bwd_tile(
         // support reaches the wave's pixels
         const int t0 = max(0, batch_end - wave_bin_final);
         const int n_work = wave_work_list(s_wmask, t0, batch_size, wave, s_list[wave]);
+        // slots t >= t_first are in front of a pixel's last contributor
+        int t_first[PX];
+#pragma unroll
+        for (int p = 0; p < PX; ++p)
+            t_first[p] = batch_end - bin_final[p];
         // One work item: Gaussian t of the batch on this wave's pixels.
         auto work_item = [&](const int t, const int col_o, const int acc_o,
                              const float4 geo,
                              const float4 con) __attribute__((always_inline)) {
-            const int32_t isect = batch_end - t;
             const float dx = geo.x - px;
             float dy[PX], sigma[PX];
             bool valid[PX];
@@ -951,7 +955,7 @@ __device__ __forceinline__ void rasterize_bwd_tile(
                 sigma[p] = gauss_sigma(con.x, con.y, con.z, dx, dy[p]);
                 // votes straight from the compares, combined in scalar
                 // registers; the selects below read the mask
-                const uint64_t valid_m = wave_ballot(isect <= bin_final[p]) &
+                const uint64_t valid_m = wave_ballot(t >= t_first[p]) &
                                          wave_ballot(sigma[p] >= 0.f) &
                                          wave_ballot(sigma[p] <= geo.w);
                 valid[p] = __builtin_amdgcn_inverse_ballot_w64(valid_m);
@@ -977,16 +981,17 @@ __device__ __forceinline__ void rasterize_bwd_tile(
                 // every contribution of theirs is selected away below
                 const float vis = portable_expf_nonpos(-sigma[p]);
                 const bool clamped = sigma[p] < con.w;
-                const float alpha = clamped ? kMaxAlpha : geo.z * vis;
                 // alpha <= 0.99, so 1 - alpha >= 0.01 (the reference's 1e-6
-                // floor never binds)
-                const float one_minus = fmaxf(kMinOneMinusAlpha, 1.f - alpha);
+                // floor never binds); an invalid pixel's is 0, which leaves
+                // its T as it is and its fac 0 (one select instead of three)
+                const float alpha = valid[p] ? (clamped ? kMaxAlpha : geo.z * vis) : 0.f;
+                const float one_minus = 1.f - alpha;
                 const float ra = __builtin_amdgcn_rcpf(one_minus);
                 const double d = (double)one_minus;
                 double r = (double)ra;
                 r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
-                T64[p] = valid[p] ? T64[p] * r : T64[p];
-                const float fac = valid[p] ? alpha * (float)T64[p] : 0.f;
+                T64[p] *= r;
+                const float fac = alpha * (float)T64[p];
                 // c . v_c: a float32 sum over many channels loses digits the
                 // cancelling difference below needs (the 32-channel conic
                 // gradient's worst element went from 2.1x to 0.5x the float32
