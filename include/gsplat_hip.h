@@ -680,7 +680,9 @@ int gsplat_rasterize_bwd(
  *   boundary of every tile, each pixel's transmittance there and the colour
  *   the next batch composited (4 * (1 + CDIM) bytes per pixel per
  *   boundary), and the list of (tile, batch) units up to each tile's last
- *   contributor.
+ *   contributor.  With more than eight channels and tiles enough to fill the
+ *   chip a unit is a whole tile, and only the transmittances are kept (4
+ *   bytes per pixel per boundary).
  * gsplat_rasterize_fwd_replay: gsplat_rasterize_fwd (render_transmittance
  *   required) that also fills the replay workspace.
  * gsplat_rasterize_bwd_replay: gsplat_rasterize_bwd with
